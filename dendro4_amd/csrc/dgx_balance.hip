@@ -15,7 +15,8 @@
 //      like a split octant in turn, in the workgroup that found it;
 //   3. k_bal_emit copies the leaves and refines, in place in the order of the
 //      curve, those that hold missing splits.
-// One host read (the number of new splits) lies between 2 and 3.  The rule's
+// One host read (the number of new splits) lies between 2 and 3, and 3 is waited
+// for.  The rule's
 // closure does not depend on the order in which splits are found, so the
 // result is the level-by-level step's, octant for octant.
 //
@@ -689,6 +690,8 @@ bool balance_search(const Key *in, size_t n, uint32_t md, int curve, hipStream_t
         else k_bal_emit<4><<<(unsigned)nblk, FB, 0, s>>>(in, n, extra.p, blk.p, base.p, hash, slots - 1, out.p);
         HIP_OK(hipGetLastError());
     }
+    // the result exists when the call returns: a hierarchy's set-up reads it on another stream
+    HIP_OK(hipStreamSynchronize(s));
     if (bs.levels) bs.leaves = total;
     if (stats) *stats = bs;
     return true;

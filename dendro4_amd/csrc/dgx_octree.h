@@ -186,7 +186,8 @@ void p2o_leaf_emit(const LeafTiles &w, const Key *pk, size_t n, uint32_t md, Key
                    hipStream_t s);
 DevBuf<Key> p2o_build(const double *d_xyz, size_t n, uint32_t md, uint32_t max_num_pts, int curve, hipStream_t s,
                       P2OStats *stats, const double *glens = nullptr);
-// Sorted leaf keys of the minimal 2:1 (face, edge, corner) balanced refinement.
+// Sorted leaf keys of the minimal 2:1 (face, edge, corner) balanced refinement,
+// written when the call returns (s has been waited for).
 DevBuf<Key> balance_build(const Key *in, size_t n, uint32_t md, int curve, hipStream_t s, BalStats *stats);
 // The same for a complete, sorted, linear octree, by searching for the splits it
 // lacks (dgx_balance.hip).  Returns false, with out untouched, for any other
