@@ -443,18 +443,25 @@ inline unsigned grid_for(size_t n, unsigned block) { return (unsigned)((n + bloc
 // Bits [begin_bit, end_bit) of the 128-bit value (hi:lo) are sorted, one pass
 // per 8-bit digit position that overlaps the range; positions in which every
 // key agrees are detected and skipped on the device.  Nothing is read back:
-// the sort is stream-ordered.  At most 8192 keys are sorted in one workgroup.
-// With level_byte the level (bits 0-4) is sorted on first.
-void radix_sort_keys(Key *keys, size_t n, hipStream_t s, int begin_bit = 0, int end_bit = 128,
-                     bool level_byte = false);
+// the sort is stream-ordered.  At most 8192 keys are sorted in one workgroup, on
+// all their bits whatever the range: keys that the range does not tell apart
+// must be equal or of no order.
+void radix_sort_keys(Key *keys, size_t n, hipStream_t s, int begin_bit = 0, int end_bit = 128);
 // Sort of keys (whole key order) through their top bits: as many passes of 8 or
 // 9 bits as n distinct keys need with some to spare, then the runs of keys that agree
-// in all those bits.  A run of more than 4096 keys is left as it is and sets
-// *fail (device word, cleared by the caller), after which the caller sorts with
-// radix_sort_keys.  Stream-ordered; nothing is read back.
+// in all those bits.  Stream-ordered; nothing is read back.  Keys that this does not
+// suit are left for sort_keys_again, and *fail (device word, cleared by the caller)
+// says why (bits): their top bits hardly spread them, and they are in no order at all
+// (kTopSkipped, with may_skip); only the runs listed in huge (count cleared by the
+// caller) are out of order (kTopHuge); some run is (kTopLong).
 // The unsorted keys go to input() (keys itself, or a buffer of the object that
 // makes the last pass end in keys).  A kernel that writes them may count their
 // digits on the way (hist(), top_hist_* below) and pass counted = true.
+enum : uint32_t { kTopLong = 1, kTopSkipped = 2, kTopHuge = 4, kTopAgain = 8 };
+struct HugeRuns {  // runs of more than 4096 keys
+    static constexpr uint32_t kMax = 64;
+    uint32_t at[kMax], len[kMax], count;
+};
 struct TopHist {
     uint32_t *ghist;   // counters of the lowest pass; 8 copies of 16 x 256 follow each other
     uint32_t np;       // passes: the digits of hi from bit `shift` up (0: no counting needed)
@@ -466,13 +473,21 @@ class TopSort {
     ~TopSort();
     Key *input() const;
     TopHist hist() const;
-    void sort(bool counted, uint32_t *fail);
+    int top_shift() const;  // the sorted bits begin at bit 64 + this
+    void sort(bool counted, uint32_t *fail, HugeRuns *huge = nullptr, bool may_skip = false);
 
   private:
     struct Impl;
     std::unique_ptr<Impl> p_;
     Key *keys_;
 };
+// The keys that a TopSort left, by its *fail word, huge runs and top_shift: those runs
+// alone if they are few; else all keys on their high words and the runs of equal ones,
+// or on their bits from begin_bit up.  With fail (device word, cleared by the caller)
+// nothing is read back for that: if *fail gets set, a second call with kTopAgain
+// sorts them.
+void sort_keys_again(Key *keys, size_t n, hipStream_t s, int begin_bit, uint32_t why, const HugeRuns *huge = nullptr,
+                     int top_shift = 0, uint32_t *fail = nullptr);
 constexpr uint32_t kTopWords = 5 * 512;  // of 8 passes of 8 bits or 5 of 9
 constexpr uint32_t kTopHistCopies = 8, kTopHistStride = 16 * 256;
 // Workgroup part of the counting: LDS counters h[kTopWords], the first

@@ -31,7 +31,7 @@ constexpr uint8_t F_BOUNDARY = 64, F_NODE = 128;
 enum : uint32_t {
     C_NPSEUDO,              // pseudo-octants
     C_LMAX,                 // finest level
-    C_FAIL_E, C_FAIL_P,     // a run too long for TopSort: elements, pseudo-octants
+    C_FAIL_E, C_FAIL_P,     // what TopSort left undone: elements (or they came unsorted), pseudo-octants
     C_UNRESOLVED, C_GHOST,  // node-list entries unresolved, found by the ghost scan
     C_REF_E, C_REF_P,       // octants referred to: elements, pseudo-octants
     C_NODES,                // NODE octants
@@ -373,13 +373,14 @@ std::unique_ptr<DaDevice> da_build(const Key *oct, size_t n, uint32_t md0, int c
         top.sort(true, ctr.p + C_FAIL_E);
     }
     dgx_read_back(hc, ctr.p, sizeof hc, s);
-    if (hc[C_FAIL_E]) radix_sort_keys(ekey.p, n, s, 0, 128);
+    if (hc[C_FAIL_E]) sort_keys_again(ekey.p, n, s, 0, hc[C_FAIL_E]);
     const size_t nbd = hc[C_NPSEUDO], N = n + nbd;
     DevBuf<Key> bkey(nbd, s);
     if (nbd) {
         TopSort top(bkey.p, nbd, s);
         k_da_bdy_emit<<<grid_for(n, B * BE_ITEMS), B, 0, s>>>(oct, bflag.p, n, tab, ctr.p, top.input());
         HIP_OK(hipGetLastError());
+        // the steps up to the next host read need the order of the cells: no may_skip
         top.sort(false, ctr.p + C_FAIL_P);
     }
     bflag.release();
@@ -409,8 +410,8 @@ std::unique_ptr<DaDevice> da_build(const Key *oct, size_t n, uint32_t md0, int c
         dgx_read_back(hc, ctr.p, sizeof hc, s);
         if (!hc[C_FAIL_P]) break;
         // a cell of the boundary holds more pseudo-octants than TopSort orders:
-        // sort them on all bits and do the steps again
-        radix_sort_keys(bkey.p, nbd, s, 0, 128);
+        // sort them again and redo the steps
+        sort_keys_again(bkey.p, nbd, s, 0, hc[C_FAIL_P]);
         HIP_OK(hipMemsetAsync(ctr.p, 0, C_COUNT * 4, s));
     }
     if (!keep_cells) cstart.release();

@@ -103,12 +103,12 @@ constexpr uint32_t kLeafWindow = 64;
 template <bool WINDOW, typename TL>
 __global__ void __launch_bounds__(TL::NT) k_leaf_count(const Key *__restrict__ pk, size_t n, uint32_t m, uint32_t md,
                                                    uint8_t *__restrict__ leaf, uint32_t *__restrict__ cnt,
-                                                   uint32_t *err, uint32_t *sat) {
+                                                   uint32_t *err, uint32_t *sat, const uint32_t *unsorted) {
     __shared__ Key sk[TL::N + 1 + (WINDOW ? 2 * kLeafWindow : 0)];  // points base - 1 - m ... with a window
     __shared__ uint8_t sp[WINDOW ? TL::N + 1 + kLeafWindow : 1], sl[TL::N + 1];
     __shared__ uint32_t s_scan[TL::NT / 64];
     const size_t base = (size_t)blockIdx.x * TL::N;
-    const uint32_t h = WINDOW ? m : 0;
+    const uint32_t h = WINDOW ? m : 0, none = *unsorted;
     // index q of sk is point base - 1 - h + q
     for (uint32_t q = threadIdx.x; q < TL::N + 1 + 2 * h; q += TL::NT) {
         const size_t g = base + q;  // one more than the point, plus h
@@ -118,6 +118,7 @@ __global__ void __launch_bounds__(TL::NT) k_leaf_count(const Key *__restrict__ p
         for (uint32_t q = threadIdx.x; q < TL::N + 1; q += TL::NT)
             if (base + q > 0 && base + q - 1 < n) sl[q] = leaf[base + q - 1];
     __syncthreads();
+    if (none) return;  // set by a launch before: the same for every thread
     if (WINDOW) {
         for (uint32_t q = threadIdx.x; q < TL::N + 1 + m; q += TL::NT) {  // pair (q, q + m)
             const size_t g = base + q;
@@ -276,14 +277,14 @@ LeafTiles::LeafTiles(size_t n, hipStream_t s)
 
 template <typename TL>
 static void leaf_count(LeafTiles &w, const Key *pk, size_t n, uint32_t m, uint32_t md, uint32_t *err, uint32_t *sat,
-                       hipStream_t s) {
+                       const uint32_t *unsorted, hipStream_t s) {
     if (m <= kLeafWindow) {
-        k_leaf_count<true, TL><<<w.tiles, TL::NT, 0, s>>>(pk, n, m, md, w.leaf.p, w.cnt.p, err, sat);
+        k_leaf_count<true, TL><<<w.tiles, TL::NT, 0, s>>>(pk, n, m, md, w.leaf.p, w.cnt.p, err, sat, unsorted);
     } else {
         DevBuf<uint8_t> lev(n - m, s);
         k_leaf_pairs<<<grid_for(n - m, LB), LB, 0, s>>>(pk, n, m, md, lev.p);
         k_leaf_levels<<<grid_for(n, LB), LB, 0, s>>>(n, m, lev.p, w.leaf.p);
-        k_leaf_count<false, TL><<<w.tiles, TL::NT, 0, s>>>(pk, n, m, md, w.leaf.p, w.cnt.p, err, sat);
+        k_leaf_count<false, TL><<<w.tiles, TL::NT, 0, s>>>(pk, n, m, md, w.leaf.p, w.cnt.p, err, sat, unsorted);
     }
     HIP_OK(hipGetLastError());
 }
@@ -295,9 +296,9 @@ static void leaf_emit(const LeafTiles &w, const Key *pk, size_t n, uint32_t md, 
     HIP_OK(hipGetLastError());
 }
 void p2o_leaf_count(LeafTiles &w, const Key *pk, size_t n, uint32_t m, uint32_t md, uint32_t *total, uint32_t *err,
-                    uint32_t *sat, hipStream_t s) {
-    if (n < kSmallN) leaf_count<SmallTile>(w, pk, n, m, md, err, sat, s);
-    else leaf_count<LargeTile>(w, pk, n, m, md, err, sat, s);
+                    uint32_t *sat, const uint32_t *unsorted, hipStream_t s) {
+    if (n < kSmallN) leaf_count<SmallTile>(w, pk, n, m, md, err, sat, unsorted, s);
+    else leaf_count<LargeTile>(w, pk, n, m, md, err, sat, unsorted, s);
     scan_exclusive_u32_async(w.cnt.p, w.off.p, w.tiles, total, s);
 }
 void p2o_leaf_emit(const LeafTiles &w, const Key *pk, size_t n, uint32_t md, Key *T, uint32_t *tb, uint32_t *tc,

@@ -170,7 +170,6 @@ struct BalStats {
     uint64_t levels = 0, seeds = 0, leaves = 0;
 };
 
-// Sorted leaf keys of the octree built from n points (xyz interleaved, device).
 // The textbook leaves of n sorted point keys (dgx_leaves.hip): count, then emit.
 struct LeafTiles {
     uint32_t tiles;
@@ -178,12 +177,14 @@ struct LeafTiles {
     DevBuf<uint32_t> cnt, off;   // per tile
     LeafTiles(size_t n, hipStream_t s);
 };
+// (unsorted: a device word; when set, the keys are not in order and the counts void)
 void p2o_leaf_count(LeafTiles &w, const Key *pk, size_t n, uint32_t m, uint32_t md, uint32_t *total, uint32_t *err,
-                    uint32_t *sat, hipStream_t s);
+                    uint32_t *sat, const uint32_t *unsorted, hipStream_t s);
 // tb, tc: each octant's first point, and the points of leaves at level md (both
 // null when no leaf is at level md)
 void p2o_leaf_emit(const LeafTiles &w, const Key *pk, size_t n, uint32_t md, Key *T, uint32_t *tb, uint32_t *tc,
                    hipStream_t s);
+// Sorted leaf keys of the octree built from n points (xyz interleaved, device).
 DevBuf<Key> p2o_build(const double *d_xyz, size_t n, uint32_t md, uint32_t max_num_pts, int curve, hipStream_t s,
                       P2OStats *stats, const double *glens = nullptr);
 // Sorted leaf keys of the minimal 2:1 (face, edge, corner) balanced refinement,

@@ -757,36 +757,39 @@ DevBuf<Key> p2o_build(const double *d_xyz, size_t n, uint32_t md, uint32_t m, in
     }
     DevBuf<Key> pk(n, s);
     // device counters: [0] textbook leaves nT, [1] a leaf at level md, [2] a
-    // point outside the domain, [3] overlapping leaves (internal error), [4] a run
-    // of equal top bits too long for TopSort, [5] triggers and from [6] on those
-    constexpr uint32_t kTrig = 6, kTrigCap = 1024 - kTrig;
-    DevBuf<uint32_t> ctr(kTrig + kTrigCap, s);
-    HIP_OK(hipMemsetAsync(ctr.p, 0, kTrig * sizeof(uint32_t), s));
+    // point outside the domain, [3] overlapping leaves (internal error), [4] what
+    // TopSort left undone, [5] triggers and from [6] on those
+    constexpr uint32_t kTrig = 6, kTrigCap = 1024 - kTrig, kHuge = sizeof(HugeRuns) / 4;
+    DevBuf<uint32_t> buf(kHuge + kTrig + kTrigCap, s);
+    HugeRuns *huge = reinterpret_cast<HugeRuns *>(buf.p);
+    uint32_t *const ctr = buf.p + kHuge;
+    HIP_OK(hipMemsetAsync(&huge->count, 0, (1 + kTrig) * sizeof(uint32_t), s));
     const double gx = glens ? glens[0] : 1.0, gy = glens ? glens[1] : 1.0, gz = glens ? glens[2] : 1.0;
+    int top_shift;
     {
         TopSort top(pk.p, n, s);
+        top_shift = top.top_shift();
         // more workgroups even out the work of large clouds; each flushes its counters
-        k_quantise<<<std::min(grid_for(n, B), n < (size_t(1) << 24) ? 2048u : 4096u), B, 0, s>>>(d_xyz, n, md, gx, gy, gz, tab, top.input(),
-                                                                 ctr.p + 2, top.hist());
+        k_quantise<<<std::min(grid_for(n, B), n < (size_t(1) << 24) ? 2048u : 4096u), B, 0, s>>>(
+            d_xyz, n, md, gx, gy, gz, tab, top.input(), ctr + 2, top.hist());
         HIP_OK(hipGetLastError());
-        top.sort(true, ctr.p + 4);
+        top.sort(true, ctr + 4, huge, true);
     }
     // Keys all at level md: bits 5-32 of the low word are zero by the key
-    // layout, so bits 32-127 decide the order.  Only a cell of the top bits that
-    // holds more points than TopSort takes has the keys sorted on those bits
-    // and the steps redone.
+    // layout, so bits 32-127 decide the order.  Where TopSort leaves keys out of
+    // order, they are sorted again and the leaves counted again.
     LeafTiles tiles(n, s);
     uint32_t hc[5];
-    for (bool full = false;; full = true) {
-        if (full) radix_sort_keys(pk.p, n, s, 32, 128);
-        p2o_leaf_count(tiles, pk.p, n, m, md, ctr.p, ctr.p + 3, ctr.p + 1, s);
-        dgx_read_back(hc, ctr.p, sizeof hc, s);
+    for (int round = 0;; ++round) {
+        p2o_leaf_count(tiles, pk.p, n, m, md, ctr, ctr + 3, ctr + 1, ctr + 4, s);
+        dgx_read_back(hc, ctr, sizeof hc, s);
         if (hc[2]) {
             dgx_set_error("points2Octree: coordinates must lie in [0,1)");
             throw DgxError();
         }
-        if (!hc[4] || full) break;
-        HIP_OK(hipMemsetAsync(ctr.p, 0, 5 * sizeof(uint32_t), s));
+        if (!hc[4]) break;
+        HIP_OK(hipMemsetAsync(ctr, 0, 5 * sizeof(uint32_t), s));
+        sort_keys_again(pk.p, n, s, 32, round ? (uint32_t)kTopAgain : hc[4], huge, top_shift, ctr + 4);
     }
     if (hc[3]) {
         dgx_set_error("points2Octree: internal error, non-empty leaves overlap");
@@ -805,10 +808,10 @@ DevBuf<Key> p2o_build(const double *d_xyz, size_t n, uint32_t md, uint32_t m, in
     DevBuf<uint32_t> tb(nT, s), tc(nT, s);
     p2o_leaf_emit(tiles, pk.p, n, md, T.p, tb.p, tc.p, s);
     // saturated-cell triggers, in the order of the leaves
-    k_p2o_trigger<<<grid_for(nT, B), B, 0, s>>>(T.p, tb.p, tc.p, nT, n, m, md, ctr.p + 5, ctr.p + kTrig, kTrigCap);
+    k_p2o_trigger<<<grid_for(nT, B), B, 0, s>>>(T.p, tb.p, tc.p, nT, n, m, md, ctr + 5, ctr + kTrig, kTrigCap);
     HIP_OK(hipGetLastError());
     std::vector<uint32_t> htrig(1 + kTrigCap);
-    dgx_read_back(htrig.data(), ctr.p + 5, htrig.size() * 4, s);
+    dgx_read_back(htrig.data(), ctr + 5, htrig.size() * 4, s);
     const uint32_t ntrig = htrig[0];
     st.triggers = ntrig;
     if (ntrig == 0) {
@@ -820,8 +823,8 @@ DevBuf<Key> p2o_build(const double *d_xyz, size_t n, uint32_t md, uint32_t m, in
         htrig.resize(ntrig);
     } else {
         DevBuf<uint32_t> trig(ntrig, s);
-        HIP_OK(hipMemsetAsync(ctr.p + 5, 0, 4, s));
-        k_p2o_trigger<<<grid_for(nT, B), B, 0, s>>>(T.p, tb.p, tc.p, nT, n, m, md, ctr.p + 5, trig.p, ntrig);
+        HIP_OK(hipMemsetAsync(ctr + 5, 0, 4, s));
+        k_p2o_trigger<<<grid_for(nT, B), B, 0, s>>>(T.p, tb.p, tc.p, nT, n, m, md, ctr + 5, trig.p, ntrig);
         HIP_OK(hipGetLastError());
         htrig.resize(ntrig);
         dgx_read_back(htrig.data(), trig.p, (size_t)ntrig * 4, s);
@@ -1036,8 +1039,7 @@ DevBuf<Key> balance_build(const Key *in, size_t n, uint32_t md, int curve, hipSt
     W.release();
     prevQ.release();
     const size_t total = used;
-    // Distinct leaves are never ancestor and descendant, so their keys order
-    // them; all bits are sorted only when a cell of the top bits holds too many.
+    // Distinct leaves are never ancestor and descendant, so their keys order them.
     DevBuf<uint32_t> longrun(1, s);
     HIP_OK(hipMemsetAsync(longrun.p, 0, sizeof(uint32_t), s));
     {
@@ -1048,7 +1050,7 @@ DevBuf<Key> balance_build(const Key *in, size_t n, uint32_t md, int curve, hipSt
     uint32_t hlong = 0;
     dgx_read_back(&hlong, longrun.p, sizeof hlong, s);
     if (hlong) {
-        radix_sort_keys(leaves.p, total, s, 8, 128);
+        sort_keys_again(leaves.p, total, s, 8, hlong);
         HIP_OK(hipStreamSynchronize(s));
     }
     out = std::move(leaves);

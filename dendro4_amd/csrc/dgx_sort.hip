@@ -417,6 +417,7 @@ __device__ __forceinline__ void status_store(uint64_t *p, uint64_t v) {
 // holds its input (0 = caller's, 1 = temporary), and the exclusive global
 // offset of every digit value.
 struct SortPlan {
+    uint32_t skip;  // a TopSort's keys agree in too many of its bits: no pass runs
     uint32_t active[16];
     uint32_t src[17];  // src[npass]: the buffer holding the sorted result
     uint32_t gofs[16 * 256];  // of digit d in pass j: gofs[j * 256 + d], with 9-bit digits gofs[j * 512 + d]
@@ -425,15 +426,32 @@ struct SortPlan {
 // One workgroup, one wave per candidate pass j (digit position
 // pos[j] = (packed >> 4j) & 15, of RB bits): a digit position is skipped when one digit
 // value holds all n keys; then thread 0 assigns the buffers in pass order.
+//
+// With fail (a TopSort) the number of passes that run keeps its parity, so that
+// the last one ends in the caller's buffer: one skipped digit gets its pass if
+// need be.  With may_skip, keys whose top bits do not spread them are left
+// unsorted and *fail is raised at once: the caller sorts them on more bits, and
+// passes over these would come on top (points in a cell of 2^-13, or half of the
+// points there).  The spread is judged by the digits' collision probabilities,
+// -sum log2 sum (c / n)^2 bits if they were independent, against the log2 n that
+// distinct places need.  Clouds of 20,000 to 128M points: uniform 17 to 25 bits more,
+// log-normal 15 to 23, 4 and 16 Gaussians of sigma 0.005 and up 10 to 20 (each with
+// hardly two keys to a run); one Gaussian of sigma 0.005 1 to 8 (up to 1.4 other
+// keys in a key's run), of 0.001 -6 to 2 (up to 170), clouds with half of their
+// points in a cell of 2^-13 -9 to -2 (hundreds to 400,000).  The line lies where runs of
+// a few keys begin.
+constexpr float kMinSpare = 2.0f;
 template <int RB>
 __global__ void __launch_bounds__(1024) k_sort_plan(const uint32_t *ghist, uint32_t n, uint64_t packed, int npass,
-                                                    SortPlan *plan) {
+                                                    SortPlan *plan, uint32_t *fail, bool may_skip) {
     __shared__ uint32_t act[16];
+    __shared__ float s_bits[16];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (w < npass) {
         const uint32_t p = (uint32_t)(packed >> (4 * w)) & 15u;
         constexpr int Q = (1 << RB) / 64;
         uint32_t c[Q], sum = 0;
+        double sq = 0.0;
         bool whole = false;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -442,7 +460,9 @@ __global__ void __launch_bounds__(1024) k_sort_plan(const uint32_t *ghist, uint3
             for (int x = 0; x < GH_COPIES; ++x) c[q] += ghist[x * (16 * 256) + (p << RB) + lane * Q + q];
             sum += c[q];
             whole = whole || c[q] == n;
+            sq += (double)c[q] * (double)c[q];
         }
+        for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
         const bool trivial = __ballot(whole) != 0;
         uint32_t total;
         uint32_t ex = wave_excl_sum(sum, total);
@@ -451,11 +471,30 @@ __global__ void __launch_bounds__(1024) k_sort_plan(const uint32_t *ghist, uint3
             plan->gofs[(w << RB) + lane * Q + q] = ex;
             ex += c[q];
         }
-        if (lane == 0) act[w] = trivial ? 0u : 1u;
+        if (lane == 0) {
+            act[w] = trivial ? 0u : 1u;
+            s_bits[w] = -log2f((float)(sq / ((double)n * (double)n)));
+        }
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t src = 0;
+        uint32_t src = 0, skipped = 0;
+        float bits = -log2f((float)n);
+        for (int j = 0; j < npass; ++j) {
+            skipped += act[j] ^ 1u;
+            bits += s_bits[j];
+        }
+        const bool none = fail && may_skip && bits < kMinSpare;
+        plan->skip = none ? 1u : 0u;
+        if (none) *fail = kTopSkipped;
+        for (int j = 0; j < npass; ++j) {
+            if (none) {
+                act[j] = 0;
+            } else if (fail && (skipped & 1u) && !act[j]) {
+                act[j] = 1;
+                skipped = 0;
+            }
+        }
         for (int j = 0; j < npass; ++j) {
             plan->active[j] = act[j];
             plan->src[j] = src;
@@ -597,129 +636,113 @@ __global__ void k_sort_finish(Key *ka, const Key *kb, size_t n, int npass, const
 
 // ---- keys sorted on their top bits: runs of equal top bits -----------------
 // After the passes over the top bits, the keys that agree in all of them (a
-// run) are put in order of the whole key.  Every position keeps its top bits
-// whatever the order inside its run, so a wave finds run borders by the top
-// bits alone while other waves reorder theirs, and only the wave that holds a
-// run's first key touches the run.  Runs of up to 8 keys inside a wave are
-// sorted by one lane each, in registers; longer ones, and those that cross the
-// end of the wave, by the wave: lane l ranks keys l, l + 64, ... against the
-// run.  Runs past kRunCap go to a list for k_sort_long_runs.  When the passes
-// left the keys in the other buffer, they are copied on the way.
-constexpr uint32_t kRunCap = 256, kRunQ = kRunCap / 64, kLongRun = 4096;
+// run) are put in order of the whole key, in place.  Every position keeps its
+// top bits whatever the order inside its run, so run borders are found by the
+// top bits alone while other workgroups reorder theirs, and only the workgroup
+// that holds a run's first key touches the run.  Where all runs are pairs inside
+// a wave, their first lanes order them.  Other workgroups put their keys (and, if
+// their last run goes on, the kRunCap behind) into LDS, and every key of a run
+// counts the keys of it that come before.  Runs past kRunCap go to a list for
+// k_sort_long_runs.
+// (A network in registers for runs of up to 8 inside a wave, and a wave per longer
+// run, which counted from global memory, run after run, took 1.93 ms in points2Octree
+// for 8M points of a Gaussian of sigma 0.001, now 1.08, and 1.08 ms for 4M in a cell
+// of 2^-6, now 0.63; 0.75 ms on 128M points of 16 Gaussians, now 0.72; 53 us on 14M
+// octants of 4 Gaussians, whose runs are siblings, now 66.)
+constexpr uint32_t kRunCap = 256, kLongRun = 4096;
 
-__device__ __forceinline__ void key_order(Key &a, Key &b) {
-    const bool sw = key_lt(b, a);
-    const Key lo = sw ? b : a, hi = sw ? a : b;
-    a = lo;
-    b = hi;
-}
-
-__global__ void __launch_bounds__(SB) k_sort_runs(const Key *ka, const Key *kb, Key *out, size_t n, int sh,
-                                                  const SortPlan *plan, int npass, uint32_t *nlong, uint32_t *list) {
-    const Key *in = plan->src[npass] ? kb : ka;
-    const bool copy = in != out;
-    const size_t j = (size_t)blockIdx.x * SB + threadIdx.x;
-    const uint32_t lane = threadIdx.x & 63;
+// skip: the plan's word (nullptr: none).  When set, the keys are still in `from`,
+// unsorted: they are copied to k if that is another buffer, and nothing else.
+__global__ void __launch_bounds__(SB) k_sort_runs(Key *k, const Key *from, size_t n, int sh, const uint32_t *skip,
+                                                  uint32_t *nlong, uint32_t *list) {
+    static_assert(kRunCap == SB, "one key behind the tile per thread");
+    constexpr uint32_t SPAN = SB + kRunCap, NW = SB / 64;
+    __shared__ Key sk[SPAN];
+    __shared__ uint64_t s_head[SPAN / 64];  // bit q: key q begins a run, or lies past the end
+    __shared__ uint32_t s_over;             // the last run of the tile goes on behind it
+    const size_t base = (size_t)blockIdx.x * SB, j = base + threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const bool in_range = j < n;
+    if (skip && *skip) {
+        if (from != k && in_range) k[j] = from[j];
+        return;
+    }
     // one load per key; the neighbours' top bits come from the adjacent lanes,
     // and from memory at the ends of the wave
-    const bool in_range = j < n;
-    const Key key = in_range ? in[j] : Key{0ull, 0ull};
+    const Key key = in_range ? k[j] : Key{0ull, 0ull};
     const uint64_t h = key.hi >> sh;
     uint64_t hp = __shfl_up(h, 1), hn = __shfl_down(h, 1);
-    if (lane == 0 && j > 0 && j <= n) hp = in[j - 1].hi >> sh;
-    if (lane == 63 && j + 1 < n) hn = in[j + 1].hi >> sh;
+    if (lane == 0 && j > 0 && j <= n) hp = k[j - 1].hi >> sh;
+    if (lane == 63 && j + 1 < n) hn = k[j + 1].hi >> sh;
     const bool next = j + 1 < n && hn == h, prev = in_range && j > 0 && hp == h;
-    if (copy && in_range && !next && !prev) out[j] = key;
     const bool start = next && !prev;
-    const uint64_t eq = __ballot(next);
-    uint64_t starts = __ballot(start);
-    if (!starts) return;
-    // the run is keys j .. j + c
-    const uint32_t c = start ? (uint32_t)__ffsll(~(unsigned long long)(eq >> lane)) - 1 : 0u;
-    const bool cross = start && lane + c >= 64, mine = start && !cross && c < 8;
-    if (mine && c == 1) {
-        Key a = key, b = in[j + 1];
-        if (copy || key_lt(b, a)) {
-            key_order(a, b);
-            out[j] = a;
-            out[j + 1] = b;
+    const uint64_t eq = __ballot(next), heads = __ballot(!prev);
+    const bool pair = start && lane < 63 && !((eq >> (lane + 1)) & 1ull);
+    if (!__syncthreads_or(start && !pair)) {
+        const Key b{__shfl_down(key.hi, 1), __shfl_down(key.lo, 1)};
+        if (pair && key_lt(b, key)) {
+            k[j] = b;
+            k[j + 1] = key;
         }
+        return;
     }
-    if (__ballot(mine && c > 1)) {
-        if (mine && c > 1) {
-            Key v[8];
-#pragma unroll
-            for (uint32_t q = 0; q < 8; ++q) v[q] = q <= c ? in[j + q] : Key{~0ull, ~0ull};
-            // Batcher's odd-even merge network for 8
-            key_order(v[0], v[1]); key_order(v[2], v[3]); key_order(v[4], v[5]); key_order(v[6], v[7]);
-            key_order(v[0], v[2]); key_order(v[1], v[3]); key_order(v[4], v[6]); key_order(v[5], v[7]);
-            key_order(v[1], v[2]); key_order(v[5], v[6]);
-            key_order(v[0], v[4]); key_order(v[1], v[5]); key_order(v[2], v[6]); key_order(v[3], v[7]);
-            key_order(v[2], v[4]); key_order(v[3], v[5]);
-            key_order(v[1], v[2]); key_order(v[3], v[4]); key_order(v[5], v[6]);
-#pragma unroll
-            for (uint32_t q = 0; q < 8; ++q)
-                if (q <= c) out[j + q] = v[q];
-        }
+    sk[threadIdx.x] = key;
+    if (lane == 0) s_head[wid] = heads;
+    if (threadIdx.x == SB - 1) s_over = next ? 1u : 0u;
+    __syncthreads();
+    const bool over = s_over;
+    const size_t jo = j + SB;
+    if (over) {
+        const Key o = jo < n ? k[jo] : Key{~0ull, ~0ull};
+        const uint64_t ho = o.hi >> sh;
+        uint64_t hq = __shfl_up(ho, 1);
+        if (lane == 0) hq = k[min(jo, n) - 1].hi >> sh;
+        sk[SB + threadIdx.x] = o;
+        const uint64_t m = __ballot(jo >= n || hq != ho);
+        if (lane == 0) s_head[NW + wid] = m;
+        __syncthreads();
     }
-    starts &= ~__ballot(mine);
-    const size_t wbase = j - lane;
-    while (starts) {
-        const uint32_t sl = (uint32_t)__ffsll((unsigned long long)starts) - 1;
-        starts &= starts - 1;
-        const size_t j0 = wbase + sl;
-        const uint64_t h0 = __shfl(h, (int)sl);
-        size_t e = n;  // run end: the first key past j0 with other top bits
-        bool ended = false;
-        size_t cpos = j0 + 1;
-        for (; cpos < n; cpos += 64) {
-            const size_t idx = cpos + lane;
-            const uint64_t other = __ballot(idx < n && (in[idx].hi >> sh) != h0);
-            if (other) {
-                e = cpos + (size_t)__ffsll((unsigned long long)other) - 1;
-                ended = true;
-                break;
-            }
-            if (cpos + 64 - j0 > kRunCap) break;
-        }
-        if (!ended && cpos >= n) ended = true;
-        if (!ended || e - j0 > kRunCap) {
-            if (lane == 0) list[atomicAdd(nlong, 1u)] = (uint32_t)j0;
-            if (copy)
-                for (size_t i = j0 + lane;; i += 64) {
-                    const bool in_run = i < n && (in[i].hi >> sh) == h0;
-                    if (in_run) out[i] = in[i];
-                    if (__ballot(!in_run)) break;
-                }
+    const uint32_t span = over ? SPAN : SB;
+    for (uint32_t q = threadIdx.x; q < span; q += SB) {
+        if (base + q >= n) continue;
+        // the run of key q: [s, e)
+        uint32_t w = q >> 6;
+        uint64_t m = s_head[w] & (~0ull >> (63 - lane));
+        while (!m && w > 0) m = s_head[--w];
+        if (!m) continue;  // begins before the tile
+        const uint32_t s0 = 64 * w + 63 - (uint32_t)__clzll(m);
+        if (s0 >= SB) continue;  // begins behind it
+        w = q >> 6;
+        m = lane == 63 ? 0ull : s_head[w] & (~0ull << (lane + 1));
+        while (!m && ++w < span / 64) m = s_head[w];
+        const uint32_t e0 = m ? 64 * w + (uint32_t)__ffsll((unsigned long long)m) - 1 : span, len = e0 - s0;
+        if (len > kRunCap) {  // so is one that goes on at SPAN, wherever it ends
+            if (q == s0) list[atomicAdd(nlong, 1u)] = (uint32_t)(base + s0);
             continue;
         }
-        const uint32_t len = (uint32_t)(e - j0);
-        Key v[kRunQ];
-        uint32_t r[kRunQ];
-#pragma unroll
-        for (uint32_t q = 0; q < kRunQ; ++q) {
-            const uint32_t t = lane + 64 * q;
-            v[q] = t < len ? in[j0 + t] : Key{0ull, 0ull};
-            r[q] = 0;
-        }
-        for (uint32_t t = 0; t < len; ++t) {
-            const Key w = in[j0 + t];
-#pragma unroll
-            for (uint32_t q = 0; q < kRunQ; ++q)
-                r[q] += (key_lt(w, v[q]) || (key_eq(w, v[q]) && t < lane + 64 * q)) ? 1u : 0u;
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < kRunQ; ++q)
-            if (lane + 64 * q < len) out[j0 + r[q]] = v[q];
+        if (len < 2) continue;
+        const Key v = sk[q];
+        uint32_t r = 0;
+#pragma unroll 4
+        for (uint32_t t = s0; t < e0; ++t) r += (key_lt(sk[t], v) || (key_eq(sk[t], v) && t < q)) ? 1u : 0u;
+        if (s0 + r != q) k[base + s0 + r] = v;
     }
 }
 
 // Runs past kRunCap, one workgroup each (bitonic in LDS).  A run past kLongRun
-// sets *fail: the caller then sorts the keys on all their bits.
-__global__ void __launch_bounds__(1024) k_sort_long_runs(Key *k, size_t n, int sh, const uint32_t *nlong,
-                                                         const uint32_t *list, uint32_t *fail) {
+// is left as it is: it is listed in huge if that is given and has room
+// (*fail |= kTopHuge), else *fail |= kTopLong.  So is everything when there are so
+// many runs that passes over more bits cost less.
+__global__ void __launch_bounds__(1024) k_sort_long_runs(Key *k, size_t n, int sh, const uint32_t *skip,
+                                                         const uint32_t *nlong, const uint32_t *list, uint32_t *fail,
+                                                         HugeRuns *huge) {
     __shared__ Key sk[kLongRun];
+    if (skip && *skip) return;
     const uint32_t nl = *nlong;
+    if (nl > 64 && nl > n / 1024) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(fail, kTopLong);
+        return;
+    }
     for (uint32_t b = blockIdx.x; b < nl; b += gridDim.x) {
         const size_t j0 = list[b];
         const uint64_t h0 = k[j0].hi >> sh;
@@ -736,7 +759,20 @@ __global__ void __launch_bounds__(1024) k_sort_long_runs(Key *k, size_t n, int s
         }
         const size_t end = j0 + len;
         if (!whole && end < n && (k[end].hi >> sh) == h0) {
-            if (threadIdx.x == 0) atomicOr(fail, 1u);
+            if (threadIdx.x == 0) {
+                size_t lo = end + 1, hi = n;  // the run's end: the keys are in order of their top bits
+                while (lo < hi) {
+                    const size_t mid = lo + (hi - lo) / 2;
+                    if ((k[mid].hi >> sh) <= h0) lo = mid + 1;
+                    else hi = mid;
+                }
+                const uint32_t at = huge ? atomicAdd(&huge->count, 1u) : HugeRuns::kMax;
+                if (at < HugeRuns::kMax) {
+                    huge->at[at] = (uint32_t)j0;
+                    huge->len[at] = (uint32_t)(lo - j0);
+                }
+                atomicOr(fail, at < HugeRuns::kMax ? kTopHuge : kTopLong);
+            }
             __syncthreads();
             continue;
         }
@@ -826,7 +862,7 @@ static void check_sort_size(size_t n) {
     }
 }
 
-void radix_sort_keys(Key *keys, size_t n, hipStream_t s, int begin_bit, int end_bit, bool level_byte) {
+void radix_sort_keys(Key *keys, size_t n, hipStream_t s, int begin_bit, int end_bit) {
     if (n < 2) return;
     check_sort_size(n);
     if (n <= kBlockSort) {
@@ -835,7 +871,7 @@ void radix_sort_keys(Key *keys, size_t n, hipStream_t s, int begin_bit, int end_
     }
     std::vector<int> passes;
     for (int p = 0; p < 16; ++p)
-        if (!(8 * p + 8 <= begin_bit || 8 * p >= end_bit) || (p == 0 && level_byte)) passes.push_back(8 * p);
+        if (!(8 * p + 8 <= begin_bit || 8 * p >= end_bit)) passes.push_back(8 * p);
     run_passes(keys, n, passes, s);
 }
 
@@ -881,15 +917,16 @@ struct PassSpace {
         }
     }
 };
-// The passes over keys kp (temporary kt), counted in w.ghist.
-void launch_passes(PassSpace &w, Key *kp, Key *kt, const std::vector<int> &passes, hipStream_t s) {
+// The passes over keys kp (temporary kt), counted in w.ghist.  fail, may_skip: as in k_sort_plan.
+void launch_passes(PassSpace &w, Key *kp, Key *kt, const std::vector<int> &passes, hipStream_t s,
+                   uint32_t *fail = nullptr, bool may_skip = false) {
     const size_t n = w.n;
     const int np = w.np, nt = w.nt;
     SortPlan *plan = w.plan;
     uint64_t *status = w.status;
     uint32_t *ctr = w.ctr;
-    if (w.rb == 9) k_sort_plan<9><<<1, 1024, 0, s>>>(w.ghist, (uint32_t)n, w.packed, np, plan);
-    else k_sort_plan<8><<<1, 1024, 0, s>>>(w.ghist, (uint32_t)n, w.packed, np, plan);
+    if (w.rb == 9) k_sort_plan<9><<<1, 1024, 0, s>>>(w.ghist, (uint32_t)n, w.packed, np, plan, fail, may_skip);
+    else k_sort_plan<8><<<1, 1024, 0, s>>>(w.ghist, (uint32_t)n, w.packed, np, plan, fail, may_skip);
     HIP_OK(hipGetLastError());
     uint32_t *fault = fault_word();
     const unsigned grid = (unsigned)w.ntiles;
@@ -922,6 +959,17 @@ void run_passes(Key *keys, size_t n, const std::vector<int> &passes, hipStream_t
 
 }  // namespace
 
+namespace {
+// Runs of keys that agree above bit 64 + sh put in order.  nlong: a zeroed word.
+void order_runs(Key *keys, const Key *from, size_t n, int sh, const uint32_t *skip, uint32_t *nlong, uint32_t *list,
+                uint32_t *fail, HugeRuns *huge, hipStream_t s) {
+    k_sort_runs<<<grid_for(n, SB), SB, 0, s>>>(keys, from, n, sh, skip, nlong, list);
+    const unsigned g = (unsigned)std::min<size_t>(512, std::max<size_t>(64, n >> 14));
+    k_sort_long_runs<<<g, 1024, 0, s>>>(keys, n, sh, skip, nlong, list, fail, huge);
+    HIP_OK(hipGetLastError());
+}
+}  // namespace
+
 struct TopSort::Impl {
     size_t n;
     hipStream_t s;
@@ -945,9 +993,7 @@ TopSort::TopSort(Key *keys, size_t n, hipStream_t s) : p_(new Impl()), keys_(key
     // 8 (a key's top bit is 0 and left out).  A pass is bound by its 32 bytes a key:
     // 504 us at 64M keys with 8 bits, 561 with 9, whose runs are shorter; with the
     // counting and balancing, 16 Gaussians of 64M points take 6.51 ms instead of
-    // 6.83, 16M points 1.81 instead of 1.89.  The 45 bits sorted then are two fewer
-    // than the six bytes hold: one cloud of 8M points and sigma 0.001, past what the
-    // 18 bits allow for, takes 2.27 ms instead of 2.10 for its longer runs.
+    // 6.83, 16M points 1.81 instead of 1.89.
     const int np9 = (int)(lg + 18 + 8) / 9;
     if (lg >= 20 && np9 < np && np9 <= 5) {
         for (int j = 0; j < np9; ++j) p_->passes.push_back(127 - 9 * np9 + 9 * j);
@@ -961,6 +1007,7 @@ TopSort::TopSort(Key *keys, size_t n, hipStream_t s) : p_(new Impl()), keys_(key
 }
 TopSort::~TopSort() {}
 // An odd number of passes ends in the other buffer, so it starts there.
+int TopSort::top_shift() const { return p_->w ? p_->passes[0] - 64 : 0; }
 Key *TopSort::input() const { return p_->w && (p_->w->np & 1) ? p_->tmp.p : keys_; }
 TopHist TopSort::hist() const {
     if (!p_->w) return TopHist{nullptr, 0, 0, 0};
@@ -968,7 +1015,7 @@ TopHist TopSort::hist() const {
     return TopHist{w.ghist + (w.rb == 8 ? (p_->passes[0] / 8) * 256 : 0), (uint32_t)w.np,
                    (uint32_t)(p_->passes[0] - 64), (uint32_t)w.rb};
 }
-void TopSort::sort(bool counted, uint32_t *fail) {
+void TopSort::sort(bool counted, uint32_t *fail, HugeRuns *huge, bool may_skip) {
     if (p_->n < 2) return;
     if (!p_->w) {
         sort_block(keys_, p_->n, p_->s);
@@ -978,9 +1025,32 @@ void TopSort::sort(bool counted, uint32_t *fail) {
     Key *a = input(), *b = a == keys_ ? p_->tmp.p : keys_;
     if (!counted)
         k_top_hist<<<(unsigned)std::min<size_t>(grid_for(p_->n, SB * GH_U), 1024), SB, 0, p_->s>>>(a, p_->n, hist());
-    launch_passes(w, a, b, p_->passes, p_->s);
-    const int sh = p_->passes[0] - 64;
-    k_sort_runs<<<grid_for(p_->n, SB), SB, 0, p_->s>>>(a, b, keys_, p_->n, sh, w.plan, w.np, w.extra, p_->list.p);
-    k_sort_long_runs<<<64, 1024, 0, p_->s>>>(keys_, p_->n, sh, w.extra, p_->list.p, fail);
-    HIP_OK(hipGetLastError());
+    launch_passes(w, a, b, p_->passes, p_->s, fail, may_skip);
+    order_runs(keys_, a, p_->n, top_shift(), &w.plan->skip, w.extra, p_->list.p, fail, huge, p_->s);
+}
+
+void sort_keys_again(Key *keys, size_t n, hipStream_t s, int begin_bit, uint32_t why, const HugeRuns *huge,
+                     int top_shift, uint32_t *fail) {
+    if (n < 2) return;
+    if (why == kTopHuge && huge) {
+        HugeRuns h;
+        dgx_read_back(&h, huge, sizeof h, s);
+        // some 60 us each, against ten passes over all keys
+        if (h.count <= std::min<size_t>(HugeRuns::kMax, std::max<size_t>(4, n >> 19))) {
+            for (uint32_t r = 0; r < h.count; ++r)
+                radix_sort_keys(keys + h.at[r], h.len[r], s, begin_bit, 64 + top_shift);
+            return;
+        }
+    }
+    if (n > kBlockSort && why != kTopAgain) {
+        DevBuf<uint32_t> w(2 + n / kRunCap + 1, s);  // long runs, fail, list
+        HIP_OK(hipMemsetAsync(w.p, 0, 8, s));
+        radix_sort_keys(keys, n, s, 64, 128);
+        order_runs(keys, keys, n, 0, nullptr, w.p, w.p + 2, fail ? fail : w.p + 1, nullptr, s);
+        if (fail) return;
+        uint32_t left = 0;
+        dgx_read_back(&left, w.p + 1, 4, s);
+        if (!left) return;
+    }
+    radix_sort_keys(keys, n, s, begin_bit, 128);
 }
