@@ -447,6 +447,13 @@ inline unsigned grid_for(size_t n, unsigned block) { return (unsigned)((n + bloc
 // all their bits whatever the range: keys that the range does not tell apart
 // must be equal or of no order.
 void radix_sort_keys(Key *keys, size_t n, hipStream_t s, int begin_bit = 0, int end_bit = 128);
+// A pass's tiles: keys per thread, and threads by the number of keys and the bits of
+// a digit.  Larger tiles mean fewer look-back steps and fewer barriers per key,
+// smaller ones more workgroups for small sorts; digits of 9 bits have one kernel.
+constexpr int kSortItems = 8;
+constexpr int sort_threads(size_t n, int digit_bits) {
+    return digit_bits == 9 || n >= (size_t(1) << 20) ? 1024 : n >= (size_t(1) << 18) ? 512 : 256;
+}
 // Sort of keys (whole key order) through their top bits: as many passes of 8 or
 // 9 bits as n distinct keys need with some to spare, then the runs of keys that agree
 // in all those bits.  Stream-ordered; nothing is read back.  Keys that this does not

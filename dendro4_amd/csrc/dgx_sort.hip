@@ -21,8 +21,7 @@
 namespace {
 
 constexpr int SB = 256;          // threads per block
-constexpr int SITEMS = 8;        // keys per thread per tile
-constexpr int STILE = SB * SITEMS;
+constexpr int SITEMS = kSortItems;  // keys per thread per tile
 
 template <int RB = 8>
 __device__ __forceinline__ uint32_t digit_of(const Key &k, int bit) {
@@ -878,14 +877,6 @@ void radix_sort_keys(Key *keys, size_t n, hipStream_t s, int begin_bit, int end_
 
 namespace {
 
-// Threads per tile: larger tiles mean fewer look-back steps and fewer
-// barriers per key, smaller ones more workgroups for small sorts.
-int sort_threads(size_t n) {
-    if (n >= (size_t(1) << 20)) return 1024;
-    if (n >= (size_t(1) << 18)) return 512;
-    return 256;
-}
-
 // Workspace of one sort of rb-bit digits, zeroed by one fill: GH_COPIES x 16 x 256 global
 // counters, 16 tile counters, the look-back status words and `extra` words for
 // the caller; then the plan.
@@ -899,8 +890,8 @@ struct PassSpace {
     uint32_t pmask = 0;
     uint64_t packed = 0;
     PassSpace(size_t n_, const std::vector<int> &passes, int rb_, size_t nextra, hipStream_t s)
-        : np((int)passes.size()), nt(sort_threads(n_)), rb(rb_), n(n_) {
-        ntiles = (n + (size_t)nt * SITEMS - 1) / ((size_t)nt * SITEMS);
+        : np((int)passes.size()), nt(sort_threads(n_, rb_)), rb(rb_), n(n_) {
+        ntiles = (n + (size_t)nt * kSortItems - 1) / ((size_t)nt * kSortItems);
         const size_t off_status = (GH_COPIES * 16 * 256 * 4 + 16 * 4 + nextra * 4 + 255) / 256 * 256;
         const size_t off_plan = off_status + (ntiles << rb) * sizeof(uint64_t);
         ws.alloc(off_plan + sizeof(SortPlan), s);
@@ -1006,8 +997,8 @@ TopSort::TopSort(Key *keys, size_t n, hipStream_t s) : p_(new Impl()), keys_(key
     p_->list.alloc(n / kRunCap + 1, s);
 }
 TopSort::~TopSort() {}
-// An odd number of passes ends in the other buffer, so it starts there.
 int TopSort::top_shift() const { return p_->w ? p_->passes[0] - 64 : 0; }
+// An odd number of passes ends in the other buffer, so it starts there.
 Key *TopSort::input() const { return p_->w && (p_->w->np & 1) ? p_->tmp.p : keys_; }
 TopHist TopSort::hist() const {
     if (!p_->w) return TopHist{nullptr, 0, 0, 0};
