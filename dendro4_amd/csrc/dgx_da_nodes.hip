@@ -275,12 +275,20 @@ __device__ void block_bitonic(V *a, uint32_t P) {
 constexpr uint32_t HS = 2048, kProbes = 64;
 constexpr uint64_t kEmpty = ~0ull;
 constexpr uint32_t kPending = 0xfffffffeu, kNone = 0xffffffffu;
+// The octants are read four at a time, 16 bytes that have to lie on a multiple of 16.
+union PointTable {
+    unsigned long long point[HS];
+    uint32_t octant[2 * HS];
+    uint4 octant4[HS / 2];
+};
+static_assert(alignof(PointTable) == 16 && sizeof(PointTable) == 8 * HS, "one table of HS slots");
 __global__ void __launch_bounds__(NB) k_da_nodes(NodeArgs A, SfcPacked tab) {
     __shared__ CurveTables T;
-    __shared__ unsigned long long hkey[HS];  // points; then owner << 16 | slot of the used ones, sorted
+    __shared__ PointTable table;             // points; then the octants outside the block that they refer to
+    unsigned long long *hkey = table.point;
     __shared__ uint32_t hown[HS];            // local index of the NODE octant anchored there
     __shared__ uint16_t hloc[HS];            // used; then the local index in the block's list
-    __shared__ uint16_t plist[HS];           // slots to be searched for
+    __shared__ uint16_t plist[HS];           // slots to be searched for; then those of the octants
     __shared__ uint32_t wf[NB / 64], wh[NB / 64], s_n, s_below, s_bad;
     const uint32_t t = threadIdx.x, lane = t & 63u, b = blockIdx.x;
     const size_t e0 = (size_t)b * NB, e = e0 + t;
@@ -436,7 +444,7 @@ __global__ void __launch_bounds__(NB) k_da_nodes(NodeArgs A, SfcPacked tab) {
     // The octants the elements refer to, in order: those of the block follow
     // their elements; the others, which lie before or after the block, are
     // ranked by counting (a bitonic sort of all took 13 us of a workgroup's 53).
-    uint32_t *own_l = reinterpret_cast<uint32_t *>(hkey);  // the points are no longer needed
+    uint32_t *own_l = table.octant;  // the points are no longer needed
     const bool in = valid && hloc[anchor] && hown[anchor] == (uint32_t)e;
     const uint64_t bin = __ballot(in);
     if (lane == 0) wf[t >> 6] = (uint32_t)__popcll(bin);
@@ -476,7 +484,7 @@ __global__ void __launch_bounds__(NB) k_da_nodes(NodeArgs A, SfcPacked tab) {
         const uint32_t i = i0 + (t >> 1);
         const uint32_t o = i < nout ? own_l[i] : 0u;
         uint32_t r = 0;
-        const uint4 *l4 = reinterpret_cast<const uint4 *>(own_l);
+        const uint4 *l4 = table.octant4;
         for (uint32_t q = t & 1u; q < npad / 4; q += 2) {
             const uint4 v = l4[q];
             r += (v.x < o ? 1u : 0u) + (v.y < o ? 1u : 0u) + (v.z < o ? 1u : 0u) + (v.w < o ? 1u : 0u);
