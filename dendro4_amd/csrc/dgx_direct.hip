@@ -636,8 +636,8 @@ __global__ void __launch_bounds__(MB) k_cgr_rows(const uint32_t *__restrict__ ni
         return;
     }
     uint32_t *out = cand + 8 * (size_t)q0;
-    if (deg == 0) {  // an interior node of no element keeps its diagonal
-        if (lane == 0) rlen[i] = 0;
+    if (deg == 0) {  // a DA's nodes are those that its elements refer to
+        if (lane == 0) atomicOr(err, 2u);
         return;
     }
     const uint32_t mine = lane < deg ? inc[q0 + lane] : kNoId;
@@ -1231,7 +1231,8 @@ CoarseInputs coarse_graph(const DaDevice &d, hipStream_t s) {
     uint32_t h[3];
     dgx_read_back(h, res, sizeof h, s);
     if (h[2]) {
-        dgx_set_error("coarse solver: a node with more than %u elements (octree not 2:1 balanced)", kMaxInc);
+        if (h[2] & 2u) dgx_set_error("coarse solver: an interior node of no element");
+        else dgx_set_error("coarse solver: a node with more than %u elements (octree not 2:1 balanced)", kMaxInc);
         throw DgxError();
     }
     in.ni = h[0];
