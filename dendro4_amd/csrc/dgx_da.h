@@ -79,6 +79,17 @@ __device__ __forceinline__ void child_frame(uint32_t v[8], uint32_t c) {
     }
 }
 
+// Slot of rank r among n: ranks r, r+1, ..., r+7 (one sibling group in SFC
+// order) go to 8 different rows of a row-major 8-row layout, so the 64 lanes of
+// one instruction hold elements from 64 different sibling groups, which in the
+// child frame touch 64 different nodes at each vertex (no LDS address conflicts).
+__device__ __forceinline__ uint32_t spread8(uint32_t r, uint32_t n) {
+    const uint32_t row = r & 7u, col = r >> 3;
+    uint32_t base = 0;
+    for (uint32_t i = 0; i < row; ++i) base += (n - i + 7u) >> 3;  // length of row i
+    return base + col;
+}
+
 // Parts of the build (dgx_da_nodes.hip).  da_flag_nodes sets the NODE flags of
 // anchors that do not hang; da_node_lists fills nlist, mask, meta, lconn and cmeta,
 // marks every octant that an element refers to (isnode) and leaves each

@@ -30,7 +30,6 @@ constexpr uint8_t F_BOUNDARY = 64, F_NODE = 128;
 // Device counters of a build.
 enum : uint32_t {
     C_NPSEUDO,              // pseudo-octants
-    C_LMAX,                 // finest level
     C_FAIL_E, C_FAIL_P,     // what TopSort left undone: elements (or they came unsorted), pseudo-octants
     C_UNRESOLVED, C_GHOST,  // node-list entries unresolved, found by the ghost scan
     C_REF_E, C_REF_P,       // octants referred to: elements, pseudo-octants
@@ -53,14 +52,14 @@ __device__ inline uint32_t n_pseudo(uint32_t f) {
 // of the embedded root, both two levels per table read.  An octant touches the
 // positive x boundary iff the x bit of all its Morton digits is 1 (TreeNode::
 // isBoundaryOctant(POSITIVE), TreeNode.cpp:247-269); bflag[i] gets the three
-// axes, ctr the number of pseudo-octants that follow and the finest level.  With
+// axes, ctr the number of pseudo-octants that follow.  With
 // unsorted, *unsorted is raised by an octant that comes before its predecessor.
 // Bound: LDS latency, 8 waves a SIMD.
 __global__ void __launch_bounds__(B) k_da_embed(const Key *in, size_t n, SfcPacked tab, Key *dkey, uint8_t *bflag,
                                                 uint32_t *ctr, uint32_t *unsorted, TopHist th) {
     __shared__ uint8_t s_rc[192], s_mc[192];
     __shared__ uint16_t s_rc2[24 * 64], s_mc2[24 * 64];
-    __shared__ uint32_t h[kTopWords], s_lmax, s_np;
+    __shared__ uint32_t h[kTopWords], s_np;
     for (uint32_t i = threadIdx.x; i < 192; i += B) {
         s_rc[i] = tab.rc[i];
         s_mc[i] = tab.mc[i];
@@ -70,10 +69,10 @@ __global__ void __launch_bounds__(B) k_da_embed(const Key *in, size_t n, SfcPack
         s_mc2[i] = rc2_entry(tab.mc, i);  // the same composition of two table steps
     }
     for (uint32_t i = threadIdx.x; i < top_hist_words(th); i += B) h[i] = 0;
-    if (threadIdx.x == 0) s_lmax = s_np = 0;
+    if (threadIdx.x == 0) s_np = 0;
     __syncthreads();
     const uint32_t root = s_rc[0];  // child 0 of the embedded root: rank | rotation << 3
-    uint32_t lm = 0, np = 0;
+    uint32_t np = 0;
     const size_t stride = (size_t)gridDim.x * B, nround = (n + stride - 1) / stride * stride;  // whole waves stay in the loop
     for (size_t i = (size_t)blockIdx.x * B + threadIdx.x; i < nround; i += stride) {
         Key k{0ull, 0ull};
@@ -102,24 +101,13 @@ __global__ void __launch_bounds__(B) k_da_embed(const Key *in, size_t n, SfcPack
             bflag[i] = (uint8_t)all;
             if (unsorted && i && key_lt(o, in[i - 1])) atomicOr(unsorted, 1u);
             np += n_pseudo(all);
-            lm = max(lm, l);
         }
         top_hist_add(h, th, k.hi, i < n);
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        lm = max(lm, (uint32_t)__shfl_xor(lm, o, 64));
-        np += (uint32_t)__shfl_xor(np, o, 64);
-    }
-    if (__lane_id() == 0) {
-        atomicMax(&s_lmax, lm);
-        atomicAdd(&s_np, np);
-    }
+    for (int o = 32; o > 0; o >>= 1) np += (uint32_t)__shfl_xor(np, o, 64);
+    if (__lane_id() == 0 && np) atomicAdd(&s_np, np);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        if (s_lmax > __hip_atomic_load(&ctr[C_LMAX], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMax(&ctr[C_LMAX], s_lmax);
-        if (s_np) atomicAdd(&ctr[C_NPSEUDO], s_np);
-    }
+    if (threadIdx.x == 0 && s_np) atomicAdd(&ctr[C_NPSEUDO], s_np);
     top_hist_flush(h, th);
 }
 
@@ -457,15 +445,6 @@ namespace {
 
 constexpr uint32_t ID_MASK = 0x3fffffffu, BDY_BIT = 0x40000000u, SHARED_BIT = 0x80000000u, NO_SLOT = 0xffffffffu;
 
-// Slot of rank r among n: ranks r, r+1, ..., r+7 (one sibling group in SFC
-// order) go to 8 different rows of a row-major 8-row layout.  As in the node
-// lists (dgx_da_nodes.hip), which place the elements' records by it.
-__device__ __forceinline__ uint32_t slot_of_rank(uint32_t r, uint32_t n) {
-    const uint32_t row = r & 7u, col = r >> 3;
-    uint32_t base = 0;
-    for (uint32_t i = 0; i < row; ++i) base += (n - i + 7u) >> 3;  // length of row i
-    return base + col;
-}
 // Turns the blocks' lists of octants into node ids, which follow the order of
 // the octants (bit 30: a Dirichlet boundary node), counts the blocks of each
 // node, and writes the elements' node ids (conn) from the block's local
@@ -507,8 +486,8 @@ __global__ void __launch_bounds__(kElemBlock) k_blk_nodes(const uint32_t *ulist,
         nflat += wf[w];
     }
     const uint64_t lt = (1ull << lane) - 1ull;
-    const uint32_t slot = hang ? nflat + slot_of_rank(ph + (uint32_t)__popcll(bh & lt), nb - nflat)
-                               : slot_of_rank(pf + (uint32_t)__popcll(bf & lt), nflat);
+    const uint32_t slot = hang ? nflat + spread8(ph + (uint32_t)__popcll(bh & lt), nb - nflat)
+                               : spread8(pf + (uint32_t)__popcll(bf & lt), nflat);
     const uint4 r = *reinterpret_cast<const uint4 *>(lconn + ((size_t)b * EB + slot) * 8);
     const uint32_t w[4] = {r.x, r.y, r.z, r.w}, c = (mt >> 8) & 7u;
     uint32_t v[8];
@@ -688,7 +667,7 @@ __global__ void __launch_bounds__(16 * G) k_blk_color(uint16_t *lconn, const uin
                                                      size_t ne, uint32_t eb, const uint16_t *cmeta, uint32_t *lrec) {
     constexpr uint32_t kCntWords = ((MAXE / 16) * 8 + 1) * 16 / 4;  // and a row that stays 0
     // degree, then fill position; then [lane group][colour] uses so far, one
-    // byte each (at most 128 uses per lane group), four to a word for the
+    // byte each (at most 16 uses per lane group), four to a word for the
     // atomic updates
     __shared__ __align__(16) uint32_t degcnt[MAXN > kCntWords ? MAXN : kCntWords];
     uint32_t *deg = degcnt, *cnt32 = degcnt;

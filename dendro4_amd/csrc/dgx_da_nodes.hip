@@ -159,17 +159,6 @@ __global__ void __launch_bounds__(NB) k_da_flag_nodes(const Key *__restrict__ k,
     if (t < nb && !(s_res[(t & ~63u) + first] & need)) flags[i] = (uint8_t)(fl | F_NODE);
 }
 
-// Slot of rank r among n: ranks r, r+1, ..., r+7 (one sibling group in SFC
-// order) go to 8 different rows of a row-major 8-row layout, so the 64 lanes of
-// one instruction hold elements from 64 different sibling groups, which in the
-// child frame touch 64 different nodes at each vertex (no LDS address conflicts).
-__device__ __forceinline__ uint32_t spread8(uint32_t r, uint32_t n) {
-    const uint32_t row = r & 7u, col = r >> 3;
-    uint32_t base = 0;
-    for (uint32_t i = 0; i < row; ++i) base += (n - i + 7u) >> 3;  // length of row i
-    return base + col;
-}
-
 struct NodeArgs {
     const Key *k;
     size_t n, ne;
