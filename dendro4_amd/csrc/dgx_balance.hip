@@ -16,9 +16,10 @@
 //   3. k_bal_emit copies the leaves and refines, in place in the order of the
 //      curve, those that hold missing splits.
 // One host read (the number of new splits) lies between 2 and 3, and 3 is waited
-// for.  The rule's
-// closure does not depend on the order in which splits are found, so the
-// result is the level-by-level step's, octant for octant.
+// for.  Where 1 or 2 find that this path cannot answer, its other workgroups stop
+// and the levels are rebuilt.  The rule's closure does not depend on the order in
+// which splits are found, so the result is the level-by-level step's, octant for
+// octant.
 //
 // Bound: the chains of dependent reads of the searches (about log2 of a cell's
 // leaves) and of the curve encodes, hidden by many waves; 32 B per leaf of
@@ -41,15 +42,18 @@ struct BalFast {
     uint32_t nnew;      // splits the input lacks
     uint32_t ntail;     // new splits that did not fit their workgroup's queue
     uint32_t lmax, lup;        // finest level; 31 minus the coarsest
-    uint32_t pad;
+    uint32_t ndense;           // workgroups that found many new splits
     unsigned long long seeds;  // what the level-by-level step counts as its seeds
+    uint32_t spread[64][16];   // levels beside leaf 0's (BS_*): 64 copies, each in a line of its own
 };
 enum : uint32_t {
     BF_INCOMPLETE = 1,  // not a complete, sorted, linear octree
     BF_HASH = 2,        // the hash set or the overflow list is full
     BF_DEEP = 4,        // a missing split more than kMaxRel levels below its leaf
-    BF_WIDE = 8         // a leaf with more than kMaxSplits missing splits
+    BF_WIDE = 8,        // a leaf with more than kMaxSplits missing splits
+    BF_MANY = 16        // the octree would grow several times over
 };
+enum : uint32_t { BS_FAR = 1, BS_FINER = 2, BS_COARSER = 4 };  // two levels or more, one finer, one coarser
 // A missing split is a 64-bit word: the leaf that holds it, and below it a 1
 // followed by its digits from the leaf's level on (3 bits a level).
 constexpr uint32_t kMaxRel = 10;
@@ -84,6 +88,8 @@ __device__ __forceinline__ void cell_end(const Key &k, uint64_t &hi, uint64_t &l
 // counts of new splits per leaf (extra) and per workgroup of k_bal_emit (blk).
 // The level range of a workgroup goes to levels[] (finest << 8 | coarsest) for
 // k_bal_find_tail: an atomic per wave on one word took 95 us of 109 on 1.9M leaves.
+// Whether there are leaves two levels apart at all is in st->spread, where most
+// workgroups find their bits set (with 8 copies for 64 this cost 20 us on 1.9M leaves).
 __global__ void __launch_bounds__(FB) k_bal_check(const Key *__restrict__ k, size_t n, uint32_t md, uint32_t cl, uint32_t bsh,
                                                   uint32_t *__restrict__ cstart, uint16_t *__restrict__ extra,
                                                   uint32_t *__restrict__ blk, uint16_t *__restrict__ levels,
@@ -92,7 +98,12 @@ __global__ void __launch_bounds__(FB) k_bal_check(const Key *__restrict__ k, siz
     const size_t i = (size_t)blockIdx.x * FB + threadIdx.x;
     const uint32_t ncell = 1u << (3 * cl);
     bool bad = false;
-    uint32_t lmax = 0, lmin = 31;
+    uint32_t lmax = 0, lmin = 31, l0 = 0, had = 0;
+    uint32_t *sp = st->spread[blockIdx.x % 64];
+    if (threadIdx.x == 0) {
+        l0 = key_level(k[0]);
+        had = __hip_atomic_load(sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     if (i < n) {
         const Key a = k[i];
         uint64_t eh, el;
@@ -125,6 +136,9 @@ __global__ void __launch_bounds__(FB) k_bal_check(const Key *__restrict__ k, siz
             lmin = min(lmin, s_lv[w][1]);
         }
         levels[blockIdx.x] = (uint16_t)(lmax << 8 | lmin);
+        const uint32_t bits = (max(lmax, l0) - min(lmin, l0) >= 2 ? BS_FAR : 0u) | (lmax > l0 ? BS_FINER : 0u) |
+                              (lmin < l0 ? BS_COARSER : 0u);
+        if (i < n && (bits & ~had)) atomicOr(sp, bits);
     }
     if (i < ncell) {
         const uint64_t h = (uint64_t)i << (63 - 3 * cl);
@@ -192,7 +206,7 @@ struct FindArgs {
     unsigned long long *tab;
     uint64_t mask;
     unsigned long long *tail;  // overflow list of new splits
-    uint32_t tail_cap;
+    uint32_t tail_cap, dense_cap;
     BalFast *st;
     uint32_t md, cl, bsh;
 };
@@ -219,8 +233,9 @@ __device__ __forceinline__ bool nbr_parent(const Axes &q, uint32_t t, uint32_t m
 
 // The octant at level lev anchored at c is required to be split.  Returns its
 // word when it was not and this call is the first to record it, else 0.
+// stop is set when this path cannot answer.
 __device__ __forceinline__ uint64_t require_split(const FindArgs &A, const uint16_t *rc2, const uint8_t *rc,
-                                                  const uint32_t c[3], uint32_t lev) {
+                                                  const uint32_t c[3], uint32_t lev, volatile uint32_t &stop) {
     uint32_t rot;
     const Key pk = morton_to_curve_rot(rc2, rc, morton_encode(c[0], c[1], c[2], lev, A.md), rot);
     // the leaf that holds its first cell: the last one not after it
@@ -238,6 +253,7 @@ __device__ __forceinline__ uint64_t require_split(const FindArgs &A, const uint1
     const uint32_t r = lev - lf;
     if (r > kMaxRel) {
         atomicOr(&A.st->flags, (uint32_t)BF_DEEP);
+        stop = 1;
         return 0;
     }
     uint32_t path = 1;
@@ -245,14 +261,26 @@ __device__ __forceinline__ uint64_t require_split(const FindArgs &A, const uint1
     const uint64_t word = (uint64_t)f << 32 | path;
     const int got = hash_insert(A.tab, A.mask, word);
     if (got <= 0) {
-        if (got < 0) atomicOr(&A.st->flags, (uint32_t)BF_HASH);
+        if (got < 0) {
+            atomicOr(&A.st->flags, (uint32_t)BF_HASH);
+            stop = 1;
+        }
         return 0;
     }
-    // one 16-bit count per leaf, two to a word
-    uint32_t *w = (uint32_t *)A.extra + (f >> 1);
-    const uint32_t sh = 16 * (f & 1u);
-    if (((atomicAdd(w, 1u << sh) >> sh) & 0xffffu) >= kMaxSplits) atomicOr(&A.st->flags, (uint32_t)BF_WIDE);
-    atomicAdd(&A.blk[f >> A.bsh], 1u);
+    // One 16-bit count per leaf, two to a word.  The lanes that name the first one's
+    // leaf or workgroup add together: a fine surface against one coarse leaf counts
+    // all its splits on one word (8.5M leaves, 9.5 ms until each was counted).
+    const uint32_t f0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)f), b0 = f0 >> A.bsh;
+    const uint64_t leaf = __ballot(f == f0), group = __ballot(f >> A.bsh == b0), lt = (1ull << __lane_id()) - 1ull;
+    if (f != f0 || !(leaf & lt)) {
+        const uint32_t sh = 16 * (f & 1u), add = f == f0 ? (uint32_t)__popcll(leaf) : 1u;
+        const uint32_t was = atomicAdd((uint32_t *)A.extra + (f >> 1), add << sh) >> sh & 0xffffu;
+        if (was + add > kMaxSplits) {
+            atomicOr(&A.st->flags, (uint32_t)BF_WIDE);
+            stop = 1;
+        }
+    }
+    if (f >> A.bsh != b0 || !(group & lt)) atomicAdd(&A.blk[f >> A.bsh], f >> A.bsh == b0 ? (uint32_t)__popcll(group) : 1u);
     return word;
 }
 
@@ -262,8 +290,19 @@ struct FindShared {
     uint16_t rc2[24 * 64];
     Axes q[FB];                   // the split octants of this round
     unsigned long long queue[2][kQueue];
-    uint32_t nnext, seeds, nnew;
+    uint32_t nnext, seeds, nnew, dense;
+    uint32_t stop;           // read between barriers only
+    volatile uint32_t halt;  // set at any time: look-ups are pointless
 };
+
+__device__ __forceinline__ uint32_t flags_now(const FindArgs &A) {
+    return __hip_atomic_load(&A.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// New splits that make a workgroup dense.  When one in 8 is, the octree would grow
+// to several times its size, on which sorting whole levels is the faster way (a
+// million points along a line, 9 times: 34 ms here before the hash set was full,
+// 35 ms there); the others then stop.
+constexpr uint32_t dense_splits(uint32_t leaves) { return leaves / 2; }
 
 __device__ __forceinline__ void find_init(FindShared &S, const SfcPacked &tab) {
     for (uint32_t i = threadIdx.x; i < 192; i += FB) {
@@ -272,7 +311,8 @@ __device__ __forceinline__ void find_init(FindShared &S, const SfcPacked &tab) {
     }
     for (uint32_t i = threadIdx.x; i < 24 * 64; i += FB) S.rc2[i] = rc2_entry(tab.rc, i);
     if (threadIdx.x == 0) {
-        S.nnext = S.seeds = S.nnew = 0;
+        S.nnext = S.seeds = S.nnew = S.dense = 0;
+        S.stop = S.halt = 0;
     }
 }
 
@@ -294,26 +334,34 @@ __device__ __forceinline__ void find_push(FindShared &S, const FindArgs &A, uint
 // Counts those inside the domain (the seeds of the level-by-level step).
 __device__ void find_round(FindShared &S, const FindArgs &A, uint32_t n, uint32_t dst) {
     uint32_t seeds = 0;
-    for (uint32_t j = threadIdx.x; j < n * 8; j += FB) {
+    for (uint32_t j = threadIdx.x; j < n * 8 && !S.halt; j += FB) {
         const Axes q = S.q[j / 8];
         uint32_t c[3];
         if (!nbr_parent(q, j % 8, A.md, c)) continue;
         ++seeds;
         if (q.lev < 2) continue;  // the parent is the root
-        find_push(S, A, require_split(A, S.rc2, S.rc, c, q.lev - 1), dst);
+        find_push(S, A, require_split(A, S.rc2, S.rc, c, q.lev - 1, S.halt), dst);
     }
     for (int o = 32; o > 0; o >>= 1) seeds += (uint32_t)__shfl_xor(seeds, o, 64);
     if ((threadIdx.x & 63u) == 0 && seeds) atomicAdd(&S.seeds, seeds);
 }
 
-// Works through `n` new splits at src until no more follow from them.
-__device__ void find_drain(FindShared &S, const FindArgs &A, uint32_t cur) {
+// Works through the new splits in queue[cur] until no more follow from them, or
+// some workgroup has found that this path cannot answer.  many: dense_splits.
+__device__ void find_drain(FindShared &S, const FindArgs &A, uint32_t cur, uint32_t many) {
     for (;;) {
         __syncthreads();
-        const uint32_t n = min(S.nnext, kQueue);
+        const uint32_t n = S.stop ? 0u : min(S.nnext, kQueue);
         __syncthreads();
         if (!n) break;
-        if (threadIdx.x == 0) S.nnext = 0;
+        if (threadIdx.x == 0) {
+            S.nnext = 0;
+            S.stop = flags_now(A);
+            if (S.nnew > many && !S.dense) {
+                S.dense = 1;
+                if (atomicAdd(&A.st->ndense, 1u) + 1 == A.dense_cap) atomicOr(&A.st->flags, (uint32_t)BF_MANY);
+            }
+        }
         for (uint32_t b = 0; b < n; b += FB) {
             const uint32_t m = min(n - b, FB);
             __syncthreads();
@@ -379,12 +427,12 @@ __device__ void find_first(FindShared &S, const FindArgs &A, uint32_t n, uint16_
     if ((threadIdx.x & 63u) == 0 && seeds) atomicAdd(&S.seeds, seeds);
     __syncthreads();
     const uint32_t m = *ntodo;
-    for (uint32_t i = threadIdx.x; i < m; i += FB) {
+    for (uint32_t i = threadIdx.x; i < m && !S.halt; i += FB) {
         const uint32_t j = todo[i];
         const Axes q = S.q[j / 7];
         uint32_t c[3];
         nbr_parent(q, 1 + j % 7, A.md, c);
-        find_push(S, A, require_split(A, S.rc2, S.rc, c, q.lev - 1), 0);
+        find_push(S, A, require_split(A, S.rc2, S.rc, c, q.lev - 1, S.halt), 0);
     }
 }
 // LPT leaves per thread.  The split octants whose first leaf lies in the
@@ -398,10 +446,17 @@ __global__ void __launch_bounds__(FB) k_bal_find(FindArgs A, size_t n, SfcPacked
     __shared__ uint32_t s_nint;
     __shared__ uint16_t s_todo[7 * FB];
     static_assert((NL - 1) / 7 + 31 < FB, "split octants of one workgroup fit one round");
-    if (A.st->flags & BF_INCOMPLETE) return;  // set by the launch before: the same for every thread
+    uint32_t sp = threadIdx.x < 64 ? A.st->spread[threadIdx.x][0] : 0u, fl = threadIdx.x == 0 ? flags_now(A) : 0u;
     find_init(S, tab);
-    if (threadIdx.x == 0) s_nint = 0;
+    for (int o = 32; o > 0; o >>= 1) sp |= (uint32_t)__shfl_xor((int)sp, o, 64);
+    if (threadIdx.x == 0) {
+        s_nint = 0;
+        // leaves of two neighbouring levels lack nothing
+        if (fl || (!(sp & BS_FAR) && (sp & (BS_FINER | BS_COARSER)) != (BS_FINER | BS_COARSER))) S.stop = 1;
+        if (S.stop) seeds[2 * (size_t)blockIdx.x] = seeds[2 * (size_t)blockIdx.x + 1] = 0;
+    }
     __syncthreads();
+    if (S.stop) return;
     const size_t i0 = (size_t)blockIdx.x * NL;
     for (uint32_t e = 0; e < LPT; ++e) {
         const uint32_t j = e * FB + threadIdx.x;
@@ -424,7 +479,7 @@ __global__ void __launch_bounds__(FB) k_bal_find(FindArgs A, size_t n, SfcPacked
     }
     __syncthreads();
     find_first(S, A, ni, s_todo, &s_nint);
-    find_drain(S, A, 0);
+    find_drain(S, A, 0, dense_splits(NL));
     if (threadIdx.x == 0) {
         seeds[2 * (size_t)blockIdx.x] = S.seeds;
         seeds[2 * (size_t)blockIdx.x + 1] = S.nnew;
@@ -450,9 +505,12 @@ __global__ void __launch_bounds__(FB) k_bal_find_tail(FindArgs A, SfcPacked tab,
     __shared__ FindShared S;
     __shared__ uint32_t s_end;
     __shared__ unsigned long long s_sum[FB / 64];
-    if (A.st->flags) return;
-    if (threadIdx.x == 0) S.seeds = S.nnew = 0;
+    if (threadIdx.x == 0) {
+        S.seeds = S.nnew = 0;
+        S.stop = flags_now(A);
+    }
     __syncthreads();
+    if (S.stop) return;
     if (blockIdx.x == 0 && A.st->ntail) {
         find_init(S, tab);
         uint32_t at = 0;
@@ -462,11 +520,11 @@ __global__ void __launch_bounds__(FB) k_bal_find_tail(FindArgs A, SfcPacked tab,
                 s_end = min(__hip_atomic_load(&A.st->ntail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), A.tail_cap);
             __syncthreads();
             const uint32_t m = min(s_end - at, kQueue);
-            if (!m) break;
+            if (!m || S.stop) break;
             for (uint32_t j = threadIdx.x; j < m; j += FB) S.queue[0][j] = A.tail[at + j];
             if (threadIdx.x == 0) S.nnext = m;
             at += m;
-            find_drain(S, A, 0);
+            find_drain(S, A, 0, ~0u);
         }
     }
     __syncthreads();
@@ -662,13 +720,14 @@ bool balance_search(const Key *in, size_t n, uint32_t md, int curve, hipStream_t
     DevBuf<uint16_t> extra(n + (n & 1), s), levels(ncheck, s);
     HIP_OK(hipMemsetAsync(ws.p, 0, zero, s));
     k_bal_check<<<ncheck, FB, 0, s>>>(in, n, md, cl, bsh, cstart.p, extra.p, blk.p, levels.p, st);
-    const FindArgs A{in, cstart.p, extra.p, blk.p, hash, slots - 1, tail, tail_cap, st, md, cl, bsh};
+    const FindArgs A{in, cstart.p, extra.p, blk.p, hash, slots - 1, tail, tail_cap, std::max(16u, nfind / 8),
+                     st, md,       cl,      bsh};
     if (small) k_bal_find<1><<<nfind, FB, 0, s>>>(A, n, tab, seeds.p);
     else k_bal_find<4><<<nfind, FB, 0, s>>>(A, n, tab, seeds.p);
     k_bal_find_tail<<<std::min(64u, 1 + nfind / 1024), FB, 0, s>>>(A, tab, seeds.p, nfind, levels.p, ncheck);
     HIP_OK(hipGetLastError());
     BalFast h;
-    dgx_read_back(&h, st, sizeof h, s);
+    dgx_read_back(&h, st, offsetof(BalFast, spread), s);
     if (h.flags) return false;
     BalStats bs{};
     if (h.lmax + h.lup >= 31 + 2) {  // else the octree is returned as it is (TreeNode.cpp:929-947)
