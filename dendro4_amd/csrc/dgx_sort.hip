@@ -437,9 +437,10 @@ struct SortPlan {
 // log-normal 15 to 23, 4 and 16 Gaussians of sigma 0.005 and up 10 to 20 (each with
 // hardly two keys to a run); one Gaussian of sigma 0.005 1 to 8 (up to 1.4 other
 // keys in a key's run), of 0.001 -6 to 2 (up to 170), clouds with half of their
-// points in a cell of 2^-13 -9 to -2 (hundreds to 400,000).  The line lies where runs of
-// a few keys begin.
-constexpr float kMinSpare = 2.0f;
+// points in a cell of 2^-13 -9 to -2 (hundreds to 400,000).  Runs of some tens of
+// keys are ordered faster than more passes are made: at 0.001, 8M points (-2 bits) take
+// 0.79 ms in points2Octree, skipped 1.08; in a cell of 2^-6, 4M (1 bit) 0.44 and 0.63.
+constexpr float kMinSpare = -3.0f;
 template <int RB>
 __global__ void __launch_bounds__(1024) k_sort_plan(const uint32_t *ghist, uint32_t n, uint64_t packed, int npass,
                                                     SortPlan *plan, uint32_t *fail, bool may_skip) {
@@ -645,7 +646,7 @@ __global__ void k_sort_finish(Key *ka, const Key *kb, size_t n, int npass, const
 // k_sort_long_runs.
 // (A network in registers for runs of up to 8 inside a wave, and a wave per longer
 // run, which counted from global memory, run after run, took 1.93 ms in points2Octree
-// for 8M points of a Gaussian of sigma 0.001, now 1.08, and 1.08 ms for 4M in a cell
+// for 8M points of a Gaussian of sigma 0.001, now 0.79, and 1.08 ms for 4M in a cell
 // of 2^-6, now 0.63; 0.75 ms on 128M points of 16 Gaussians, now 0.72; 53 us on 14M
 // octants of 4 Gaussians, whose runs are siblings, now 66.)
 constexpr uint32_t kRunCap = 256, kLongRun = 4096;
