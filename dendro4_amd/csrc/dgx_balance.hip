@@ -211,6 +211,10 @@ struct FindArgs {
     uint32_t md, cl, bsh;
 };
 
+__device__ __forceinline__ uint32_t flags_now(const FindArgs &A) {
+    return __hip_atomic_load(&A.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Parent t (bit a: the neighbouring one along axis a) of the neighbours of the
 // split octant q.  False when it lies outside the domain.
 __device__ __forceinline__ bool nbr_parent(const Axes &q, uint32_t t, uint32_t md, uint32_t c[3]) {
@@ -267,6 +271,10 @@ __device__ __forceinline__ uint64_t require_split(const FindArgs &A, const uint1
         }
         return 0;
     }
+    if (flags_now(A)) {
+        stop = 1;
+        return 0;
+    }
     // One 16-bit count per leaf, two to a word.  The lanes that name the first one's
     // leaf or workgroup add together: a fine surface against one coarse leaf counts
     // all its splits on one word (8.5M leaves, 9.5 ms until each was counted).
@@ -295,9 +303,6 @@ struct FindShared {
     volatile uint32_t halt;  // set at any time: look-ups are pointless
 };
 
-__device__ __forceinline__ uint32_t flags_now(const FindArgs &A) {
-    return __hip_atomic_load(&A.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // New splits that make a workgroup dense.  When one in 8 is, the octree would grow
 // to several times its size, on which sorting whole levels is the faster way (a
 // million points along a line, 9 times: 34 ms here before the hash set was full,
@@ -706,9 +711,10 @@ bool balance_search(const Key *in, size_t n, uint32_t md, int curve, hipStream_t
     const uint32_t bsh = blk_shift(small ? 1 : 4);
     const size_t nblk = (n + (size_t(1) << bsh) - 1) >> bsh;
     // Twice as many slots as half the leaves could fill: up to n / 4 new
-    // splits (the octree nearly triples) stay under half load.
-    uint64_t slots = 4096;
-    while (slots < n / 2) slots <<= 1;
+    // splits (the octree nearly triples) stay under half load.  Small octrees get
+    // room for up to n: the other step takes some 20 launches a level whatever their size.
+    uint64_t slots = 16384;
+    while (slots < (small ? 2 * n : n / 2)) slots <<= 1;
     const uint32_t tail_cap = (uint32_t)(slots / 4);
     const size_t zero = sizeof(BalFast) + slots * 8;
     DevBuf<uint8_t> ws(zero + (size_t)tail_cap * 8, s);
@@ -720,7 +726,7 @@ bool balance_search(const Key *in, size_t n, uint32_t md, int curve, hipStream_t
     DevBuf<uint16_t> extra(n + (n & 1), s), levels(ncheck, s);
     HIP_OK(hipMemsetAsync(ws.p, 0, zero, s));
     k_bal_check<<<ncheck, FB, 0, s>>>(in, n, md, cl, bsh, cstart.p, extra.p, blk.p, levels.p, st);
-    const FindArgs A{in, cstart.p, extra.p, blk.p, hash, slots - 1, tail, tail_cap, std::max(16u, nfind / 8),
+    const FindArgs A{in, cstart.p, extra.p, blk.p, hash, slots - 1, tail, tail_cap, small ? ~0u : nfind / 8,
                      st, md,       cl,      bsh};
     if (small) k_bal_find<1><<<nfind, FB, 0, s>>>(A, n, tab, seeds.p);
     else k_bal_find<4><<<nfind, FB, 0, s>>>(A, n, tab, seeds.p);
