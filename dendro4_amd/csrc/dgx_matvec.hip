@@ -597,9 +597,11 @@ __global__ void __launch_bounds__(B, 4) k_matvec_pipe(const uint32_t *__restrict
 // to pipeline, so what counts is the chain of loads (offsets, node entries, x) and
 // the element phase of a CU that holds one workgroup.  One element and two nodes
 // per thread, eight waves, halve that phase's LDS operations per wave.  Same sums,
-// same bits.  FP32 sweeps of a 16,000-point hierarchy 5.4 -> 3.95 us; a matvec of
-// 20,000 4-Gaussian points (two launches) 7.0 -> 6.6 us.  With about 300 blocks
-// both take 8.5 us, with 600 the pipelined kernel is faster (10.5 against 11.4).
+// same bits.  FP32 sweeps of a 16,000-point hierarchy 5.4 -> 3.95 us; FP64 matvecs
+// back to back on one mesh of 4,000 to 117,000 octants (both launches) 7.3-7.5 ->
+// 6.8-7.2 us, three meshes of 20,000 points in turn in FP32 7.7-7.9 us either way.
+// With about 300 blocks both take 8.5 us, with 600 the pipelined kernel is faster
+// (10.5 against 11.4).
 constexpr uint32_t kOnceBlocks = 256;
 template <typename T, bool DIR, int EPI>
 __global__ void __launch_bounds__(kElemBlock) k_matvec_once(const uint32_t *__restrict__ rec, size_t ne,
